@@ -1,15 +1,16 @@
 // A routed feed-forward (mixers.h): every row picks a few experts by its router logits and only
 // their weights are read.  Logits, picks, weights and sums are float.
 //
-// A decode batch in bfloat16 (widths of whole lines): the picked experts' weights are streamed once for all of
-// their rows, hidden units stay float, and a last kernel adds a row's picks up (expert_stream_kernel).
-//
-// 32-bit weights, and widths that are no multiples of 64: the picked experts' hidden units (a workgroup
+// 32-bit weights, and widths that are no multiples of 8: the picked experts' hidden units (a workgroup
 // per (row, pick, 16 hidden units)); the down products with the weighted sum over a row's picks (a
 // workgroup per (row, 16 outputs)), so that a row's result is added up in one place and in a fixed
 // order.  A wave takes one weight row at a time, 16 bytes a lane, against the row's input in LDS.
 //
-// A prompt (64 rows and more, bfloat16) goes through tiles on the matrix cores: the (row, pick) pairs
+// A decode batch in bfloat16 (up to 63 rows): the picked experts' weights are read once for all of their rows,
+// and a last kernel adds a row's picks up; the same sums in the same order (expert_chains_kernel).
+// Some more rows of many experts: the like with sums in the order of the bfloat16 MFMAs (expert_stream_kernel).
+//
+// A prompt (64 rows and more of fewer experts, bfloat16) goes through tiles on the matrix cores: the (row, pick) pairs
 // are sorted by expert in one workgroup, a workgroup takes 128 pairs of one expert by 64 or 128 hidden units
 // (up to 256 outputs) through LDS with v_mfma_f32_32x32x16_bf16; the hidden units are rounded to bfloat16
 // once, as every product's input is; a last kernel adds a row's picks up in their order.  Which
@@ -608,32 +609,331 @@ __global__ __launch_bounds__(256) void grouped_sum_kernel(const float* __restric
             }
     }
     const float same = identity > 0 ? identity_weight(ids, w, top, E, identity) : 0.f;
+    float4 input = make_float4(0.f, 0.f, 0.f, 0.f);
     if (same != 0.f) {
         const uint2 hv = *(const uint2*)(h + row * D + d);
-        total.x += same * __uint_as_float(hv.x << 16);
-        total.y += same * __uint_as_float(hv.x & 0xffff0000u);
-        total.z += same * __uint_as_float(hv.y << 16);
-        total.w += same * __uint_as_float(hv.y & 0xffff0000u);
+        input = make_float4(__uint_as_float(hv.x << 16), __uint_as_float(hv.x & 0xffff0000u), __uint_as_float(hv.y << 16),
+                            __uint_as_float(hv.y & 0xffff0000u));
     }
-    *o = make_float4(before.x + total.x, before.y + total.y, before.z + total.z, before.w + total.w);
+    // (as expert_down_kernel adds up, to the bit)
+    const auto sum = [&](float b, float t, float x) { return b + t + (same != 0.f ? same * x : 0.f); };
+    *o = make_float4(sum(before.x, total.x, input.x), sum(before.y, total.y, input.y), sum(before.z, total.z, input.z), sum(before.w, total.w, input.w));
 }
 
-// ---- the same for a few rows, the experts' weights streamed once -----------------------------------------
+// ---- the same for a few rows, the experts' weights read once, to the bit -----------------------------------
 // A decode batch's picks meet in the experts: 16 rows that pick two of eight bring every expert four
 // rows.  A workgroup of four waves takes the weight rows of one expert (HIDDEN: 16 hidden units' rows of gate
-// and of up; else 32 outputs of down) for all of the expert's pairs, up to 64 at a time, so that every
-// weight is read once, past the caches.  The waves take K in turns of 64 columns; a wave's loads go straight into LDS stages
+// and of up; else 32 outputs of down) for all of the expert's pairs, up to 16 at a time, so that weights
+// are read once, past the caches.  Both operands go from memory straight into LDS, the weights into each wave's own part
+// of it (the first 512 columns before the pairs are known), the pairs' rows half a step or a step ahead.
+//
+// A pair's sums are those of the kernels above, to the bit: chain l of 64 adds the products of columns 8 l .. + 7 of
+// every 512, one after another, and the chains' sums meet by halves, quarters, ... of the 64.  A chain is a block of
+// v_mfma_f32_4x4x1_16b_f32, which does one FMA for each of four weight rows and four pairs in 16 chains: twice the rate of
+// the vector ALU.  (The bfloat16 MFMAs, four times as fast again, add several products up in an order of their own.  A
+// step's pairs are few enough for the float ones, and with other sums than a workgroup per pair has, a router behind
+// them that is not sure of a pick decides otherwise.)
+// Which pairs share an expert changes no pair's result.
+// Bound by the experts' bytes: sixteen experts of 4,096 x 4,096 at 16 rows, two picked, 238 us with the adding
+// kernel where the weights of the experts picked take 201 at 6.5 TB/s (a workgroup per pair and 16 units, which
+// read an expert's weights for every pair of its own: 742); eight of 2,048 x 2,048 47.7 us, floor 31 (203).  From eight pairs
+// an expert on the MFMAs' time shows (48 rows: hidden units 45 us, 13 of them if nothing else ran; 16 rows: 31.6).
+#define EC_LISTED 1024         // pairs of the step of which a workgroup lists its expert's at a time
+typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
+
+// One step of the meeting of a wave's sums: lanes whose bit is clear take a, the others b, each with its partner's added.
+template <int BIT>
+__device__ __forceinline__ float meet(float a, float b) {
+    if constexpr (BIT == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    } else if constexpr (BIT == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    } else {
+        const bool set = threadIdx.x & BIT;
+        const float mine = set ? b : a, theirs = set ? a : b;
+        if constexpr (BIT == 8) return mine + other_lane<0x128>(theirs);                   // a rotation of 16 by 8
+        else return mine + other_lane<0x1B>(other_lane<0x141>(theirs));                    // eight mirrored, then each four: lane ^ 7 ^ 3
+    }
+}
+// N sums of 16 groups of four lanes: group b is left with that of v[b / (16 / N)].
+template <int N, int BIT = 32>
+__device__ __forceinline__ float meet_all(float (&v)[N]) {
+    constexpr int HALF = N > 1 ? N / 2 : 1;
+    float half[HALF];
+#pragma unroll
+    for (int i = 0; i < HALF; ++i) half[i] = meet<BIT>(v[i], v[N > 1 ? i + N / 2 : i]);
+    if constexpr (BIT > 4) return meet_all<HALF, BIT / 2>(half);
+    else return half[0];
+}
+
+// all but the newest n loads have arrived, n known when compiled
+__device__ __forceinline__ void wait_until_newest(int n) {
+    switch (n) {
+#define EC_CASE(i) case i: wait_for_loads<i>(); break;
+        EC_CASE(14) EC_CASE(10) EC_CASE(9) EC_CASE(8) EC_CASE(7) EC_CASE(6) EC_CASE(5) EC_CASE(4) EC_CASE(3) EC_CASE(2) EC_CASE(1)
+#undef EC_CASE
+        default: wait_for_loads<0>(); break;      // (fewer than allowed to be on their way is always right)
+    }
+}
+
+// What a wave multiplies by: eight weight rows (HIDDEN: four of gate, four of up).  A step of 512 columns is eight pieces of a
+// kilobyte, piece 2 g + half chains 16 g .. + 15 of four of the rows, lane 4 b + i chain 16 g + b of row i.  A piece has a
+// place in LDS and the next step's is asked for when it has been read.
+struct WeightRows {
+    const bf16_t* half[2];
+    unsigned row_at[2];    // this lane's row of either half, in bytes
+    int K;
+    unsigned lds;          // of the wave's places
+    __device__ __forceinline__ void ask(int piece, int s) const {          // (past the row's end its last eight columns again)
+        const int lane = threadIdx.x % 64;
+        const unsigned at = row_at[piece % 2] + (unsigned)min(512 * s + 128 * (piece / 2) + 8 * (lane / 4), K - 8) * 2u;
+        stream_16_bytes_to_lds(at, same_in_every_lane(half[piece % 2]), lds + piece * 1024);
+    }
+};
+
+// Four PG pairs at a time; the weights' first pieces have been asked for.
+template <bool HIDDEN, int PG>
+__device__ __forceinline__ void expert_chains_body(const void* __restrict__ a, float* __restrict__ out, const WeightRows& rows, int top, int K, int N,
+                                                   const int32_t* __restrict__ picks, const ExpertAct& xa, const int32_t* pairs, int n_here, int n0,
+                                                   const char* places, const char* x, unsigned x_lds) {
+    // The pairs' rows come in units of G chains' sixteenths (a step, or half of one), a unit ahead.  A kilobyte of them is, for
+    // chains 16 g .. + 15 of four pairs, eight columns of bfloat16 or four of float; lane 4 b + j has chain 16 g + b of pair j.
+    // A unit's kilobytes are in the order [g][four pairs][first, last four columns], and every wave asks for a quarter.
+    constexpr int G = !HIDDEN && PG == 4 ? 2 : 4, UNITS = 4 / G, X_PIECES = (HIDDEN ? 1 : 2) * G * PG, X_MINE = X_PIECES / 4;
+    constexpr int PG_MINE = PG / UNITS;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64, b = lane / 4, j = lane % 4;
+    const int n_steps = (K + 511) / 512;
+    const char* x_row[PG_MINE];
+#pragma unroll
+    for (int i = 0; i < PG_MINE; ++i) {
+        const int pair = pairs[min(4 * (wave % UNITS * PG_MINE + i) + j, n_here - 1)];          // pairs past the last repeat it and are never stored
+        x_row[i] = (const char*)a + (HIDDEN ? (size_t)(pair / top) * K * 2 : (size_t)pair * K * 4);
+    }
+    auto ask_x = [&](int unit) {
+        const unsigned to = x_lds + ((unit & 1) * X_PIECES + wave * X_MINE) * 1024;
+        const int c = min(128 * (G * unit + wave / UNITS) + 8 * b, K - 8);
+#pragma unroll
+        for (int i = 0; i < PG_MINE; ++i) {
+            if constexpr (HIDDEN) {
+                gather_16_bytes_to_lds(x_row[i] + c * 2, to + i * 1024);
+            } else {
+                gather_16_bytes_to_lds(x_row[i] + c * 4, to + i * 2048);
+                gather_16_bytes_to_lds(x_row[i] + c * 4 + 16, to + i * 2048 + 1024);
+            }
+        }
+    };
+    f32x4 acc[2][PG][4];                // [half][pairs][g]: four rows of this lane's chain and pair
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int pg = 0; pg < PG; ++pg)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) acc[h][pg][g] = f32x4{0.f, 0.f, 0.f, 0.f};
+    u32x4 w;                            // this lane's 16 bytes of the piece that is next
+    float xv[PG][8];                    // and the chain's eight columns of the pairs' rows
+    auto inputs = [&](int s, int g, bool past_end) {
+        const char* from = x + ((UNITS * s + g / G & 1) * X_PIECES + g % G * (X_PIECES / G)) * 1024 + lane * 16;
+#pragma unroll
+        for (int pg = 0; pg < PG; ++pg) {
+            u32x4 lo, hi;
+            if constexpr (HIDDEN) {
+                const u32x4 v = *(const u32x4*)(from + pg * 1024);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    xv[pg][2 * e] = __uint_as_float(v[e] << 16);
+                    xv[pg][2 * e + 1] = __uint_as_float(v[e] & 0xffff0000u);
+                }
+            } else {
+                lo = *(const u32x4*)(from + pg * 2048);
+                hi = *(const u32x4*)(from + pg * 2048 + 1024);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) xv[pg][e] = __uint_as_float(lo[e]), xv[pg][4 + e] = __uint_as_float(hi[e]);
+            }
+            if (past_end)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) xv[pg][e] = 0.f;
+        }
+    };
+    auto multiply = [&](int piece) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float we = __uint_as_float(e % 2 ? w[e / 2] & 0xffff0000u : w[e / 2] << 16);
+#pragma unroll
+            for (int pg = 0; pg < PG; ++pg)
+                acc[piece % 2][pg][piece / 2] = __builtin_amdgcn_mfma_f32_4x4x1f32(we, xv[pg][e], acc[piece % 2][pg][piece / 2], 0, 0, 0);
+        }
+    };
+    ask_x(0);
+    wait_for_loads<0>();
+    __syncthreads();
+    w = *(const u32x4*)(places + lane * 16);
+    for (int s = 0; s + 1 < n_steps; ++s) {
+#pragma unroll
+        for (int piece = 0; piece < 8; ++piece) {
+            if (piece % (2 * G) == 0) {
+                // this wave's share of the unit has come: a step's is older than the piece that has been waited for, half a step's than four pieces
+                if (UNITS == 2) wait_for_loads<4>();
+                if (s + piece > 0) __syncthreads();
+                ask_x(UNITS * s + piece / (2 * G) + 1);          // into the part that has been read
+            }
+            if (piece % 2 == 0) inputs(s, piece / 2, false);
+            // The next piece comes out of LDS meanwhile: behind it six newer ones are on their way, and the rows of the units
+            // that began in the last seven turns.  (The first eight pieces have come whatever the count.)
+            wait_until_newest(6 + X_MINE * ((piece % (2 * G) <= 6) + (UNITS == 2 && piece % 4 <= 2)));
+            const u32x4 next = *(const u32x4*)(places + (piece + 1) % 8 * 1024 + lane * 16);
+            asm volatile("" : "+v"(w));          // this piece has been read: its place takes the next step's
+            rows.ask(piece, s + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(piece);
+            __builtin_amdgcn_sched_barrier(0);
+            w = next;
+        }
+    }
+#pragma unroll
+    for (int piece = 0; piece < 8; ++piece) {
+        const bool past_end = 512 * (n_steps - 1) + 128 * (piece / 2) + 8 * b >= K;
+        if (piece % (2 * G) == 0) {
+            if (piece > 0) wait_for_loads<0>();
+            else if (UNITS == 2) wait_for_loads<4>();
+            if (n_steps > 1 || piece > 0) __syncthreads();
+            if (UNITS == 2 && piece == 0) ask_x(2 * n_steps - 1);
+        }
+        if (piece % 2 == 0) inputs(n_steps - 1, piece / 2, past_end);
+        wait_until_newest(6 - piece + (UNITS == 2 && piece < 4 ? X_MINE : 0));
+        const u32x4 next = *(const u32x4*)(places + (piece + 1) % 8 * 1024 + lane * 16);          // (the last one's is not used)
+        if (past_end) w = u32x4{0, 0, 0, 0};
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(piece);
+        __builtin_amdgcn_sched_barrier(0);
+        w = next;
+    }
+    // the chains' sums: bits 5 and 4 of a chain's number are g's, the others the lane's
+    float sum[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        float v[4 * PG];
+#pragma unroll
+        for (int pg = 0; pg < PG; ++pg)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                v[4 * pg + r] = (acc[h][pg][0][r] + acc[h][pg][2][r]) + (acc[h][pg][1][r] + acc[h][pg][3][r]);
+        sum[h] = meet_all(v);
+    }
+    constexpr int SAME = 4 / PG;        // groups of four lanes with the same sum
+    const int at = b / SAME, col = 4 * (at / 4) + j, n = n0 + (HIDDEN ? 4 : 8) * wave + at % 4;
+    if (b % SAME || col >= n_here) return;
+    const int pair = pairs[col];
+    float* to = out + (size_t)pair * N + n;
+    if constexpr (HIDDEN) {
+        const float on_input = xa.weight_on_input ? ((const float*)(picks + (size_t)(pair / top) * 2 * top + top))[pair % top] : 1.f;
+        if (n < N) *to = expert_act(xa, sum[0] * on_input, sum[1] * on_input);
+    } else {
+        if (n < N) to[0] = sum[0];
+        if (n + 4 < N) to[4] = sum[1];
+    }
+}
+
+// by_pair: workgroups (., y) stand for the expert of pair y, if no earlier pair has picked it; else for expert y
+template <bool HIDDEN>
+__global__ __launch_bounds__(256, 2) void expert_chains_kernel(const void* __restrict__ a, const int32_t* __restrict__ picks, float* __restrict__ out,
+                                                               const bf16_t* __restrict__ w0, const bf16_t* __restrict__ w1, int E, int top,
+                                                               int n_pairs, int K, int N, ExpertAct xa, int by_pair) {
+    extern __shared__ __attribute__((aligned(1024))) char chains_lds[];          // the waves' places | the pairs' rows of two steps
+    __shared__ int32_t pairs[EC_LISTED];
+    __shared__ int32_t n_listed;
+    const int y = blockIdx.y;
+    const int e = by_pair ? picks[(size_t)(y / top) * 2 * top + y % top] : y;
+    if (e < 0 || e >= E) return;            // (uniform over the workgroup)
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const int n0 = blockIdx.x * (HIDDEN ? 16 : 32), first_row = n0 + (HIDDEN ? 4 : 8) * wave;
+    const unsigned lds = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) char*)chains_lds);
+    WeightRows rows;
+    rows.half[0] = w0 + ((size_t)e * N + n0) * K;
+    rows.half[1] = HIDDEN ? w1 + ((size_t)e * N + n0) * K : rows.half[0];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)             // (past the matrix its last row)
+        rows.row_at[h] = (unsigned)(min(first_row + (HIDDEN ? 0 : 4 * h) + (int)threadIdx.x % 4, N - 1) - n0) * (unsigned)K * 2u;
+    rows.K = K;
+    rows.lds = lds + wave * 8192;
+#pragma unroll
+    for (int piece = 0; piece < 8; ++piece) rows.ask(piece, 0);          // before the pairs are known
+    __builtin_amdgcn_sched_barrier(0);
+    constexpr int AT_ONCE = 16;
+    const char* places = chains_lds + wave * 8192;
+    const char* x = chains_lds + 4 * 8192;
+    bool asked = true, first_pairs = true;
+    for (int from = 0; from < n_pairs; from += EC_LISTED) {
+        if (from > 0) __syncthreads();      // the list before has been read
+        if (threadIdx.x < 64) {
+            int n = 0;
+            const int end = min(n_pairs, from + EC_LISTED);
+            for (int p0 = from; p0 < end; p0 += 256) {
+                int got[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int p = p0 + 64 * i + (int)threadIdx.x;
+                    got[i] = p < end ? picks[(size_t)(p / top) * 2 * top + p % top] : -1;
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const uint64_t mask = __ballot(got[i] == e);
+                    if (got[i] == e) pairs[n + __popcll(mask & ((1ull << threadIdx.x) - 1))] = p0 + 64 * i + (int)threadIdx.x;
+                    n += __popcll(mask);
+                }
+            }
+            if (threadIdx.x == 0) n_listed = n;
+        }
+        __syncthreads();
+        const int n = n_listed;
+        if (n == 0) continue;
+        if (first_pairs && by_pair && pairs[0] != y) break;          // (an earlier pair's workgroups have the expert)
+        first_pairs = false;
+        for (int first = 0; first < n; first += AT_ONCE) {
+            const int n_here = min(AT_ONCE, n - first);
+            if (!asked) {
+                __syncthreads();            // the pairs before have been read
+#pragma unroll
+                for (int piece = 0; piece < 8; ++piece) rows.ask(piece, 0);
+            }
+            asked = false;
+            if (n_here <= 4) expert_chains_body<HIDDEN, 1>(a, out, rows, top, K, N, picks, xa, pairs + first, n_here, n0, places, x, lds + 4 * 8192);
+            else if (n_here <= 8) expert_chains_body<HIDDEN, 2>(a, out, rows, top, K, N, picks, xa, pairs + first, n_here, n0, places, x, lds + 4 * 8192);
+            else expert_chains_body<HIDDEN, 4>(a, out, rows, top, K, N, picks, xa, pairs + first, n_here, n0, places, x, lds + 4 * 8192);
+        }
+    }
+    if (asked) wait_for_loads<0>();         // (nothing may be written to LDS that is another's by then)
+}
+
+template <bool HIDDEN>
+static int launch_expert_chains(const void* a, const int32_t* picks, float* out, const bf16_t* w0, const bf16_t* w1, int E, int top, int rows, int K,
+                                int N, const ExpertAct& xa, hipStream_t stream) {
+    const int n_pairs = rows * top, by_pair = n_pairs < E;
+    constexpr size_t lds = 64 * 1024;
+    static bool raised = false;
+    if (!raised) {
+        hipError_t e = hipFuncSetAttribute((const void*)expert_chains_kernel<HIDDEN>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        PICOLM_REQUIRE(e == hipSuccess, "routed_experts: cannot raise the LDS limit to %zu: %s", lds, hipGetErrorString(e));
+        raised = true;
+    }
+    const dim3 grid((unsigned)ceil_div(N, HIDDEN ? 16 : 32), (unsigned)(by_pair ? n_pairs : E));
+    expert_chains_kernel<HIDDEN><<<grid, 256, lds, stream>>>(a, picks, out, w0, w1, E, top, n_pairs, K, N, xa, by_pair);
+    PICOLM_LAUNCH_CHECK("routed_experts (in chains)");
+    return 0;
+}
+
+// ---- the same for some more rows: bfloat16 MFMAs -----------------------------------------------------------
+// A workgroup of four waves takes the weight rows of one expert as above, for up to 64 of the expert's pairs at a
+// time.  The waves take K in turns of 64 columns; a wave's loads go straight into LDS stages
 // of its own, a kilobyte each (as in gemm_skinny_staged_kernel of gemm_mfma.hip), weights as the first operand
 // of v_mfma_f32_16x16x32_bf16 and the pairs' rows as the second; the waves' sums meet in LDS in a fixed order.
 // The hidden units stay float: a wave takes a float's three bfloat16 parts of eight bits each, which add
 // up to it exactly, through three MFMAs, so that every product is exact and sums are float.
 // Which pairs share an expert changes no pair's result.
-// Bound by the experts' bytes: sixteen experts of 4,096 x 4,096 at 16 rows, two picked, 235 us with the adding
-// kernel where the weights of the experts picked take 201 at 6.5 TB/s (a workgroup per pair and 16 units, which
-// read an expert's weights for every pair of its own: 742); eight of 2,048 x 2,048 47 us, floor 31 (203).
+// Bound by the experts' bytes: sixteen experts of 4,096 x 4,096 at 64 rows, two picked, 263 us with the adding
+// kernel where the weights of the experts picked take 248 at 6.5 TB/s; 64 of 1,408 x 2,048, six picked, 213 us, floor 170.
 #define ES_MOST_PAIRS 512      // pairs of one expert that a workgroup lists (a row picks an expert once)
-typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
-
 // eight floats as three bfloat16 chunks: x = hi + mid + lo (a number that is not finite lies in hi alone)
 __device__ __forceinline__ void split_chunk(const f32x4& x0, const f32x4& x1, bf16x8& hi, bf16x8& mid, bf16x8& lo) {
     u32x4 h, m, l;
@@ -871,21 +1171,27 @@ static int grouped_product(const bf16_t* a, const int32_t* plan, void* out, cons
 
 #define GM_FROM_ROWS 64      // rows of a step from which the matrix cores take the experts
 
-// Whether the kernels that stream an expert's weights once take a step: bfloat16 throughout, whole lines
-// of 64 columns in both widths, aligned rows.  Below 64 rows the other choice is a workgroup per pair (16 rows, eight
-// experts of 2,048 x 2,048, two picked: 47 us against 203).  From 64 rows on it is the tiles of 128 pairs, which win
-// when an expert has more pairs than tiles of 16 take in two turns: 2,048 x 2,048, 20 pairs an expert 72 against
-// 81 us, 24 80 against 81, 48 108 against 85; sixteen experts of 4,096 x 4,096, 16 pairs an expert 317 against some 340
-// us, 24 433 against 345.
+// What either kind of kernels that read an expert's weights once needs: bfloat16 throughout, 16-byte aligned buffers and rows
+static bool reads_weights_once(const picolm_routed_experts_args* a, const picolm_step_view* v, int widths_in) {
+    return v->dtype == PICOLM_BF16 && a->weight_dt == PICOLM_BF16 && a->width % widths_in == 0 && a->ff % widths_in == 0 && v->extra[2] &&
+           (((uintptr_t)v->in | (uintptr_t)v->out | (uintptr_t)v->extra[1] | (uintptr_t)v->extra[2] | (uintptr_t)a->gate | (uintptr_t)a->up |
+             (uintptr_t)a->down) & 15) == 0;
+}
+// Below 64 rows every kernel gives a row the same bits, and the chains are the fastest that do: eight experts of 2,048 x
+// 2,048, two picked, 16 rows 47.7 us against 203 with a workgroup per pair, 32 rows 59 and 63 rows 86.  (The bfloat16 MFMAs
+// take 46 to 51 at any of these, in another order of sums.)
+static bool takes_chains(const picolm_routed_experts_args* a, const picolm_step_view* v) {
+    return v->rows < GM_FROM_ROWS && a->experts <= 65535 && (int64_t)v->rows * a->top <= 65535 && reads_weights_once(a, v, 8);
+}
+// From 64 rows on the streamed kernels, until an expert has more pairs than their tiles of 16 take in two turns; then the tiles of
+// 128 pairs win: 2,048 x 2,048, 20 pairs an expert 72 against 81 us, 24 80 against 81, 48 108 against 85; sixteen
+// experts of 4,096 x 4,096, 16 pairs an expert 317 against some 340 us, 24 433 against 345.
 #define ES_MOST_ROWS 255
 #define ES_PAIRS_AN_EXPERT 20
 static bool streams_experts(const picolm_routed_experts_args* a, const picolm_step_view* v) {
-    return v->dtype == PICOLM_BF16 && a->weight_dt == PICOLM_BF16 && a->width % 64 == 0 && a->ff % 64 == 0 && v->extra[2] &&
-           (v->rows < GM_FROM_ROWS || (v->rows <= ES_MOST_ROWS && (int64_t)v->rows * a->top <= (int64_t)ES_PAIRS_AN_EXPERT * a->experts)) &&
-           (((uintptr_t)v->in | (uintptr_t)v->out | (uintptr_t)v->extra[1] | (uintptr_t)v->extra[2] | (uintptr_t)a->gate | (uintptr_t)a->up |
-             (uintptr_t)a->down) & 15) == 0 &&
-           (int64_t)v->rows * a->top * a->ff < (1ll << 29) && (int64_t)v->rows * a->width < (1ll << 30) && 32ll * a->width < (1ll << 30) &&
-           32ll * a->ff < (1ll << 30);
+    return v->rows >= GM_FROM_ROWS && v->rows <= ES_MOST_ROWS && (int64_t)v->rows * a->top <= (int64_t)ES_PAIRS_AN_EXPERT * a->experts &&
+           reads_weights_once(a, v, 64) && (int64_t)v->rows * a->top * a->ff < (1ll << 29) && (int64_t)v->rows * a->width < (1ll << 30) &&
+           32ll * a->width < (1ll << 30) && 32ll * a->ff < (1ll << 30);
 }
 
 extern "C" int picolm_call_routed_experts(void* user, const picolm_step_view* v) {
@@ -911,12 +1217,13 @@ extern "C" int picolm_call_routed_experts(void* user, const picolm_step_view* v)
     if (v->rows <= 0) return 0;
     const int32_t* picks = (const int32_t*)v->extra[0];
     float* act = (float*)v->extra[1];
-    if (streams_experts(a, v)) {
+    const bool chains = takes_chains(a, v);
+    if (chains || streams_experts(a, v)) {
         PICOLM_REQUIRE(v->extra_row_bytes[2] >= (int64_t)top * D * 4, "routed_experts: scratch rows too short for the pairs' outputs");
         float* y = (float*)v->extra[2];
-        int rc = launch_expert_stream<true>(v->in, picks, act, (const bf16_t*)a->gate, (const bf16_t*)a->up, E, top, v->rows, D, F, xa, v->stream);
+        int rc = (chains ? launch_expert_chains<true> : launch_expert_stream<true>)(v->in, picks, act, (const bf16_t*)a->gate, (const bf16_t*)a->up, E, top, v->rows, D, F, xa, v->stream);
         if (rc) return rc;
-        rc = launch_expert_stream<false>(act, picks, y, (const bf16_t*)a->down, nullptr, E, top, v->rows, F, D, xa, v->stream);
+        rc = (chains ? launch_expert_chains<false> : launch_expert_stream<false>)(act, picks, y, (const bf16_t*)a->down, nullptr, E, top, v->rows, F, D, xa, v->stream);
         if (rc) return rc;
         grouped_sum_kernel<<<dim3(v->rows, ceil_div(D, 1024)), 256, 0, v->stream>>>(y, picks, (float*)v->out, E, top, D, a->adds, (const bf16_t*)v->in,
                                                                                    a->identity, plain_sum);

@@ -23,7 +23,7 @@ class Experts:
         w = torch.rand(rows, top, generator=self.gen, device=DEV) + 0.1
         return ids, w, torch.cat([ids, w.view(torch.int32)], 1).contiguous()
 
-    def run(self, h, words, top, out, adds):
+    def run(self, h, words, top, out, adds, streamed=True):
         from picolm_amd import kernels
         from picolm_amd.engine import program as P
         from picolm_amd.parts.calls import RoutedExpertsArgs
@@ -36,7 +36,7 @@ class Experts:
         v = P.StepView()
         v.struct_bytes, v.dtype, v.rows, v.n_tokens = ctypes.sizeof(P.StepView), 1, rows, rows
         v.inp, v.out, v.in_row_bytes, v.out_row_bytes = h.data_ptr(), out.data_ptr(), self.D * 2, self.D * 4
-        for i, t in enumerate((words, act, y, plan)):
+        for i, t in enumerate((words, act, y, plan) if streamed else (words, act)):
             v.extra[i], v.extra_row_bytes[i] = t.data_ptr(), t.shape[1] * 4
         v.stream = torch.cuda.current_stream().cuda_stream
         f = kernels.lib().picolm_call_routed_experts
@@ -86,6 +86,29 @@ def test_streamed_experts(E, D, F, rows):
     # 64 rows and more with many pairs an expert go through tiles that round the hidden units to eight bits (2^-9 each)
     streamed = rows < 64 or rows * top <= 20 * E
     assert norm < (2e-6 if streamed else 4e-3) and worst < (1e-5 if streamed else 2e-2), (E, D, F, rows, norm, worst)
+
+
+# up to four and eight pairs of an expert at a time and more of them, one expert, fewer pairs than experts; widths below 512
+# columns, that end inside 512, and inside a workgroup's weight rows
+@pytest.mark.parametrize("E,D,F", [(8, 2048, 2048), (1, 64, 64), (3, 200, 328), (40, 320, 192), (2, 1032, 2568)])
+@pytest.mark.parametrize("rows", [1, 2, 7, 16, 33, 63])
+def test_streamed_experts_are_those_of_a_workgroup_per_pair_to_the_bit(E, D, F, rows):
+    """However many of its rows a step brings an expert: the same sums in the same order, so that a router behind them that is not
+    sure of a pick decides as it did."""
+    for x, top in ((Experts(E, D, F), min(E, 2)), (Experts(E, D, F, identity=2), 3), (Experts(E, D, F, act=1, weight_on_input=1), min(E, 3))):
+        h = torch.randn(rows, D, generator=x.gen, device=DEV).bfloat16()
+        ids, w, words = x.picks(rows, top)
+        out = torch.randn(rows, D, generator=x.gen, device=DEV)
+        for adds in (True, False):
+            assert torch.equal(x.run(h, words, top, out.clone(), adds), x.run(h, words, top, out.clone(), adds, streamed=False))
+
+
+def test_streamed_experts_of_more_pairs_than_a_workgroup_lists_at_a_time():
+    x = Experts(40, 64, 64)
+    h = torch.randn(63, 64, generator=x.gen, device=DEV).bfloat16()
+    ids, w, words = x.picks(63, 20)
+    out = torch.zeros(63, 64, device=DEV)
+    assert torch.equal(x.run(h, words, 20, out.clone(), False), x.run(h, words, 20, out.clone(), False, streamed=False))
 
 
 @pytest.mark.parametrize("rows", [3, 40])
