@@ -286,10 +286,7 @@ __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_plain_mfma_kernel(AttnA
     }
     __syncthreads();
     const int tid = threadIdx.x;
-    auto put = [&](int row, int hq, int c, float m, float l, float2 o) {
-        const float inv = factor(row, hq, m, l);
-        const float* gate = gate_row(row, hq);
-        const float y0 = gated(gate, c, o.x * inv), y1 = gated(gate, c + 1, o.y * inv);
+    auto store = [&](int row, int hq, int c, float y0, float y1) {
         const size_t at = (size_t)row * (a.out_stride ? a.out_stride : a.H * DV) + (size_t)hq * DV + c;
         if (a.out_float) {
             ((float*)a.out)[at] = y0;
@@ -301,22 +298,18 @@ __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_plain_mfma_kernel(AttnA
     };
     for (int idx = tid; idx < n_rows * (DV / 2); idx += 64 * PLAIN_WAVES) {
         const int q = idx / (DV / 2), c = 2 * (idx % (DV / 2));
-        float m = NEG_BIG, l = 0.f;
-        float2 o = make_float2(0.f, 0.f);
-        float ms[PLAIN_WAVES];
+        // one wave after the other joins the first: every join has the running maximum's rounding, as a wave's tiles have
+        const float* first = merge_lds + (size_t)q * STRIDE;
+        float m = first[DV], l = first[DV + 1];
+        float2 o = *(const float2*)(first + c);
 #pragma unroll
-        for (int w = 0; w < PLAIN_WAVES; ++w) {
-            ms[w] = merge_lds[((size_t)w * n_rows + q) * STRIDE + DV];
-            m = fmaxf(m, ms[w]);
-        }
-#pragma unroll
-        for (int w = 0; w < PLAIN_WAVES; ++w) {
-            const float* row = merge_lds + ((size_t)w * n_rows + q) * STRIDE;
-            const float f = exp2_flushing(ms[w] - m);
-            const float2 v = *(const float2*)(row + c);
-            l += f * row[DV + 1];
-            o.x += f * v.x;
-            o.y += f * v.y;
+        for (int w = 1; w < PLAIN_WAVES; ++w) {
+            const float* other = merge_lds + ((size_t)w * n_rows + q) * STRIDE;
+            const float m_o = other[DV], m_new = fmaxf(m, m_o), mine_k = exp2_flushing(m - m_new), other_k = exp2_flushing(m_o - m_new);
+            const float2 v = *(const float2*)(other + c);
+            l = fmaf(l, mine_k, other[DV + 1] * other_k);
+            o = make_float2(fmaf(o.x, mine_k, v.x * other_k), fmaf(o.y, mine_k, v.y * other_k));
+            m = m_new;
         }
         const int hq = a.decode ? first_head + q : first_head, row = a.decode ? seq : first_tok + q;
         if (a.decode && n_chunks > 1) {
@@ -330,12 +323,14 @@ __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_plain_mfma_kernel(AttnA
                 *(float2*)(po + 2 + c) = o;
             }
         } else {
-            put(row, hq, c, m, l, o);
+            const float inv = factor(row, hq, m, l);
+            const float* gate = gate_row(row, hq);
+            store(row, hq, c, gated(gate, c, o.x * inv), gated(gate, c + 1, o.y * inv));
         }
     }
     if (!a.decode || n_chunks <= 1 || !a.chunks_done) return;       // (uniform over the workgroup)
     // The workgroup that finishes a sequence's last chunk reads all of them back and writes the
-    // output, chunk by chunk in their order, so that the sum does not depend on who it was; see
+    // output, so that the sum does not depend on who it was; see
     // attn_decode_mfma_kernel for why single coherent accesses and no fence.
     __shared__ int i_am_last;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // this thread's stores have been acknowledged
@@ -344,38 +339,62 @@ __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_plain_mfma_kernel(AttnA
     if (tid == 0) i_am_last = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == n_chunks - 1;
     __syncthreads();
     if (!i_am_last) return;
+    // A row's maximum and denominator first, a wave a row and a lane a chunk; then the columns: to the bit what the
+    // merge kernel (attention_generic.hip) makes of them.  The first eight chunks' columns are asked for ahead of that.
+    constexpr int EARLY = 8;
+    const size_t chunk = DV + 2;
+    const auto partial_of = [&](int q) { return a.partial + ((size_t)seq * a.H + first_head + q) * a.max_splits * chunk; };
+    float2 st[EARLY], v[EARLY];
+    auto ask = [&](int idx, int i0) {
+        const float* p = partial_of(idx / (DV / 2));
+        const int c = 2 * (idx % (DV / 2));
+#pragma unroll
+        for (int e = 0; e < EARLY; ++e) {
+            const float* pe = p + min(i0 + e, n_chunks - 1) * chunk;
+            st[e] = load_agent(pe);
+            v[e] = load_agent(pe + 2 + c);
+        }
+    };
+    if (tid < n_rows * (DV / 2)) ask(tid, 0);
+    for (int q = wave; q < n_rows; q += PLAIN_WAVES) {
+        const float* p = partial_of(q);
+        float m = NEG_BIG;
+        for (int i = lane; i < n_chunks; i += 64) m = fmaxf(m, load_agent(p + i * chunk).x);
+        float M = wave_max(m);
+        if (a.sink) M = fmaxf(M, a.sink[first_head + q]);
+        float l = 0.f;
+        for (int i = lane; i < n_chunks; i += 64) {
+            const float2 s = load_agent(p + i * chunk);
+            l += expf(s.x - M) * s.y;
+        }
+        float L = wave_sum(l);
+        if (a.sink) L += expf(a.sink[first_head + q] - M);
+        if (lane == 0) {
+            merge_lds[2 * q] = M;
+            merge_lds[2 * q + 1] = (L > 0.f ? 1.0f / L : 0.f) * (a.out_stride ? a.out_mult : 1.f);
+        }
+    }
+    __syncthreads();
     for (int idx = tid; idx < n_rows * (DV / 2); idx += 64 * PLAIN_WAVES) {
         const int q = idx / (DV / 2), c = 2 * (idx % (DV / 2)), hq = first_head + q;
-        const float* p = a.partial + ((size_t)seq * a.H + hq) * a.max_splits * (DV + 2);
-        float m = NEG_BIG, l = 0.f;
+        const float M = merge_lds[2 * q], inv = merge_lds[2 * q + 1];
         float2 o = make_float2(0.f, 0.f);
-        for (int i0 = 0; i0 < n_chunks; i0 += 8) {             // eight chunks are asked for at a time
-            float2 st[8], v[8];
+        for (int i0 = 0; i0 < n_chunks; i0 += EARLY) {
+            if (idx != tid || i0 > 0) ask(idx, i0);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float* pe = p + (size_t)min(i0 + e, n_chunks - 1) * (DV + 2);
-                st[e] = load_agent(pe);
-                v[e] = load_agent(pe + 2 + c);
-            }
-            float m_new = m;
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-                if (i0 + e < n_chunks) m_new = fmaxf(m_new, st[e].x);
-            const float kept = expf(m - m_new);
-            l *= kept;
-            o.x *= kept;
-            o.y *= kept;
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
+            for (int e = 0; e < EARLY; ++e)
                 if (i0 + e < n_chunks) {
-                    const float f = expf(st[e].x - m_new);
-                    l += f * st[e].y;
+                    const float f = expf(st[e].x - M);
                     o.x += f * v[e].x;
                     o.y += f * v[e].y;
                 }
-            m = m_new;
         }
-        put(seq, hq, c, m > 0.5f * NEG_BIG ? m * LOG2E : NEG_BIG, l, o);
+        if (a.gate) {
+            const float* gate = a.gate + (size_t)seq * a.gate_stride + (size_t)hq * (a.gate_per_head ? 1 : DV);
+            o.x *= 1.f / (1.f + expf(-gate[a.gate_per_head ? 0 : c]));
+            o.y *= 1.f / (1.f + expf(-gate[a.gate_per_head ? 0 : c + 1]));
+        }
+        store(seq, hq, c, o.x * inv, o.y * inv);
     }
     if (tid == 0) *counter = 0;          // as the next launch expects it
 }

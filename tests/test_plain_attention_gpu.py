@@ -59,6 +59,7 @@ def test_decode(H, G, d, pages_per_chunk, window):
     sink_d, gate_d = torch.from_numpy(sink).to(DEV), torch.from_numpy(gate).to(DEV)
     x = Extras(v_head_dim=d, sink=sink_d.data_ptr(), gate=gate_d.data_ptr(), gate_stride=H, gate_per_head=1)
     done = torch.zeros(K().attn_decode_counters(5, H, G), dtype=torch.int32, device=DEV)
+    merged = None
     for counters in (None, done, done):          # twice: the counters must be left at zero
         out = torch.full_like(case.q_dev, float("nan"))
         partial = torch.full((5 * H * most * (d + 2),), float("nan"), device=DEV)
@@ -67,6 +68,9 @@ def test_decode(H, G, d, pages_per_chunk, window):
             at(b.seq_pos0), at(case.table), case.table.shape[1], case.table.shape[1], H, G, d, window, ctypes.c_float(1.0 / math.sqrt(d)),
             ctypes.byref(x), at(counters), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0, lib.picolm_last_error()
         close(out, want)
+        # whoever combines the chunks, the merge kernel or the last workgroup: the same sums
+        assert merged is None or torch.equal(out, merged)
+        merged = out
     assert not done.any()
 
 
