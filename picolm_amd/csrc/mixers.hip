@@ -204,7 +204,7 @@ __global__ __launch_bounds__(1024) void qk_norm_all_store_kernel(QkPrepare a, T*
         kept[k] = i < n ? term(i) : Term{0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     }
 #pragma unroll
-    for (int k = 0; k < ROW_KEEP; ++k) ssq += kept[k].own * kept[k].own;
+    for (int k = 0; k < ROW_KEEP; ++k) ssq = fmaf(kept[k].own, kept[k].own, ssq);          // (in the loop's order below, to the bit)
     for (int i = threadIdx.x + ROW_KEEP * blockDim.x; i < n; i += blockDim.x) {
         const float y = entry(i);
         ssq += y * y;
@@ -812,7 +812,7 @@ __global__ __launch_bounds__(1024) void gated_norm_wide_kernel(const float* __re
         gk[i] = c < group ? gate_at(c) : 0.f;
     }
 #pragma unroll
-    for (int i = 0; i < ROW_KEEP; ++i) ssq += xk[i] * xk[i];
+    for (int i = 0; i < ROW_KEEP; ++i) ssq = fmaf(xk[i], xk[i], ssq);          // (in the loop's order below, to the bit)
     for (int c = threadIdx.x + ROW_KEEP * blockDim.x; c < group; c += blockDim.x) {
         const float xv = entry(c);
         ssq += xv * xv;
@@ -889,8 +889,8 @@ __global__ __launch_bounds__(1024) void normed_sum_kernel(float* __restrict__ x,
     }
 #pragma unroll
     for (int i = 0; i < ROW_KEEP; ++i) {
-        sa += ak[i] * ak[i];
-        sb += bk[i] * bk[i];
+        sa = fmaf(ak[i], ak[i], sa);          // (in the loop's order below, to the bit)
+        sb = fmaf(bk[i], bk[i], sb);
     }
     for (int c = threadIdx.x + ROW_KEEP * blockDim.x; c < W; c += blockDim.x) {
         sa += ar[c] * ar[c];

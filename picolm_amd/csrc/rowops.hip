@@ -375,7 +375,7 @@ __global__ __launch_bounds__(1024) void gated_postnorm_kernel(float* __restrict_
         const int c = threadIdx.x + i * blockDim.x;
         sk[i] = c < W ? sum_at(c) : 0.f;
         wk[i] = c < W ? weight[c] : 0.f;
-        ssq += sk[i] * sk[i];
+        ssq = fmaf(sk[i], sk[i], ssq);          // (said so: the first two squares as one expression would round the second, not the first)
     }
     for (int c = threadIdx.x + BN_KEEP * blockDim.x; c < W; c += blockDim.x) {
         const float s = sum_at(c);

@@ -120,3 +120,49 @@ def test_a_norm_over_all_heads_then_the_rotation(H, G, d, half):
     for i, (p, pg) in enumerate(zip([5, 0, 7], [2, 0, 1])):
         close(k_pages[pg, :, p, :], key[i])
         assert torch.equal(v_pages[pg, :, :, p], rows[i, (H + G) * d:].view(G, d))
+
+
+def squares_in_order(x, threads):
+    """Sums of the rows' squares [rows] as a workgroup of `threads` makes them in 32 bits: a thread's entries one after another
+    through an FMA, a wave's threads by halves, quarters, ..., the waves one after another."""
+    import numpy as np
+    rows, W = x.shape
+    padded = np.zeros((rows, -(-W // threads) * threads), np.float32)
+    padded[:, :W] = x
+    s = np.zeros((rows, threads), np.float32)
+    for part in np.split(padded, padded.shape[1] // threads, 1):
+        wide = part.astype(np.longdouble)                 # (a square and a sum of this size lie in 64 bits as they are)
+        s = (wide * wide + s).astype(np.float32)
+    s = s.reshape(rows, threads // 64, 64)
+    while s.shape[2] > 1:
+        s = s[:, :, :s.shape[2] // 2] + s[:, :, s.shape[2] // 2:]
+    total = np.zeros(rows, np.float32)
+    for w in range(threads // 64):
+        total = total + s[:, w, 0]
+    return total
+
+
+# what is kept in registers between the passes changes no bit (rows that fit, and rows that do not)
+@pytest.mark.parametrize("W", [2048, 3000, 9000])
+def test_row_norms_to_the_bit(W):
+    import numpy as np
+    from picolm_amd.parts.calls import GatedNormArgs, GatedPostnormArgs, NormedSumArgs
+    rows = 48
+    gen = torch.Generator(device=DEV).manual_seed(W)
+    x, u, w = (torch.randn(*s, generator=gen, device=DEV) for s in ((rows, W), (rows, W), (W,)))
+    xs, us, ws = (t.cpu().numpy() for t in (x, u, w))
+    fma = lambda a, b, c: (np.asarray(a, np.longdouble) * b + c).astype(np.float32)
+    f32 = np.float32
+
+    def normed_rows(rows_):
+        mean = squares_in_order(rows_, 1024) / f32(W)
+        return rows_ * (f32(1) / np.sqrt(mean + f32(1e-5)))[:, None] * ws
+    got = torch.empty_like(x)
+    call("picolm_call_gated_norm", GatedNormArgs(w.data_ptr(), W, W, W, 1e-5, 0, W, 0, 0, 0, 0, 0.0), rows, u, got)
+    assert np.array_equal(got.cpu().numpy(), normed_rows(us))
+    got = x.clone()
+    call("picolm_call_normed_sum", NormedSumArgs(w.data_ptr(), None, W, 1e-5, 0.5), rows, u, got)
+    assert np.array_equal(got.cpu().numpy(), fma(f32(0.5), normed_rows(us), xs))
+    got = x.clone()
+    call("picolm_call_gated_postnorm", GatedPostnormArgs(w.data_ptr(), None, W, 1.5, 1e-5), rows, u, got)
+    assert np.array_equal(got.cpu().numpy(), normed_rows(fma(f32(1.5), xs, us)))
