@@ -338,16 +338,13 @@ def gemm_tiled(a, w, c, epilogue: int = EPI_STORE, variant: int = 0) -> None:
 
 
 SPLITK_WS_FLOATS = 8 << 20        # 32 MB of partial sums: splits * M * N may not exceed it
-_splitk_ws: dict = {}
 
 
 def splitk_workspace(device) -> torch.Tensor:
-    """One buffer per GPU for the partial sums of products cut along K; kernels of one stream
-    run in order, so they can share it."""
-    key = torch.device(device).index or 0
-    if key not in _splitk_ws:
-        _splitk_ws[key] = torch.empty(SPLITK_WS_FLOATS, dtype=torch.float32, device=device)
-    return _splitk_ws[key]
+    """A buffer for the partial sums of one product cut along K, of the current stream's memory: hold it until the
+    product has been queued.  (Kernels of one stream run in order, so that what the allocator hands out on it next may lie
+    there; products on two streams must not share a buffer.)"""
+    return torch.empty(SPLITK_WS_FLOATS, dtype=torch.float32, device=device)
 
 
 def gemm_tiled_splitk(a, w, c, epilogue: int, variant: int, splits: int) -> None:
@@ -418,9 +415,10 @@ def gemm_linked(a, w, c, epilogue: int, prepare=None, prepared=None) -> None:
         n_parts = ssq.shape[0]
         if ssq.shape[1] != rows:
             raise KernelError("gemm_linked: the statistics are not those of this product's input rows")
+    ws = splitk_workspace(a.device)
     _check(lib().picolm_linear(_ptr(a), dt_of(a), _ptr(w), dt_of(w), _ptr(c), dt_of(c), M, N, K, epilogue,
                                _ptr(nw), _ptr(nh), _ptr(nssq), next_parts, _ptr(ssq), n_parts, int(norm_len), c_float(eps),
-                               _ptr(splitk_workspace(a.device)), _stream()))
+                               _ptr(ws), _stream()))
 
 
 def gemm(a: torch.Tensor, w: torch.Tensor, c: torch.Tensor, epilogue: int = EPI_STORE) -> None:

@@ -81,3 +81,22 @@ def test_float_product_of_a_row_does_not_depend_on_the_other_rows():
                 got = c[:M].clone()
                 kernels.gemm(a[:M].contiguous(), w, got, epi)
                 assert torch.equal(got, want[:M]), (M, N, K, epi)
+
+
+def test_float_products_on_two_streams():
+    """Products that are cut into shares at the same time on two streams: each has partial sums of its own."""
+    from picolm_amd import kernels
+    streams, work = [torch.cuda.Stream() for _ in range(2)], []
+    for i in range(2):
+        a, w, c = operands(40, 2048, 8192, 0, seed=i)
+        want = torch.empty_like(c)
+        kernels.gemm(a, w, want, 0)
+        work.append((a, w, want, [torch.empty_like(c) for _ in range(20)]))
+    torch.cuda.synchronize()
+    for k in range(20):
+        for s, (a, w, want, outs) in zip(streams, work):
+            with torch.cuda.stream(s):
+                kernels.gemm(a, w, outs[k], 0)
+    torch.cuda.synchronize()
+    for a, w, want, outs in work:
+        assert all(torch.equal(o, want) for o in outs)
