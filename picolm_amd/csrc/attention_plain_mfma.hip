@@ -71,7 +71,7 @@ __device__ __forceinline__ float2 load_agent(const float* p) {
 
 template <int D, int DV>
 __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_plain_mfma_kernel(AttnArgs a) {
-    extern __shared__ float merge_lds[];        // [PLAIN_WAVES][rows in use][DV + 4]: values, maximum and sum of each wave
+    extern __shared__ __attribute__((aligned(16))) float merge_lds[];        // [PLAIN_WAVES][rows in use][DV + 4]: values, maximum and sum of each wave
     const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, col = lane & 31, h = lane >> 5;
     const int R = a.H / a.G;
     int seq, g, head, tok, qpos, qpos_first, slot, page_lo, page_hi, hi, split = 0, n_chunks = 1, first_tile, kept_tiles;

@@ -74,7 +74,7 @@ struct Sums {
 template <int KC, int RULE>
 __global__ __launch_bounds__(256) void state_chunk_prepare_kernel(StateChunks a) {
     constexpr int KD = 16 * KC, KLD = KD + 4;
-    extern __shared__ float sc_lds[];
+    extern __shared__ __attribute__((aligned(16))) float sc_lds[];
     float* Ks = sc_lds;                      // [64][KLD]
     float* T = Ks + SC_LEN * KLD;            // [64][SC_LD]: D, then T
     float* X = T + SC_LEN * SC_LD;           // [64][SC_LD] (delta rule)
