@@ -69,16 +69,16 @@ __device__ __forceinline__ float2 load_agent(const float* p) {
     return make_float2(__uint_as_float((unsigned)bits), __uint_as_float((unsigned)(bits >> 32)));
 }
 
-template <int D, int DV>
+template <int D, int DV, bool DECODE>
 __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_plain_mfma_kernel(AttnArgs a) {
     extern __shared__ __attribute__((aligned(16))) float merge_lds[];        // [PLAIN_WAVES][rows in use][DV + 4]: values, maximum and sum of each wave
-    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, col = lane & 31, h = lane >> 5;
+    const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), col = lane & 31, h = lane >> 5;
     const int R = a.H / a.G;
     int seq, g, head, tok, qpos, qpos_first, slot, page_lo, page_hi, hi, split = 0, n_chunks = 1, first_tile, kept_tiles;
     int n_rows, first_head, first_tok = 0, work_index = 0;         // columns in use, head and token of the first
-    int early[4] = {0, 0, 0, 0};        // physical pages of a chunk's first four pages, from the work list
+    int early0 = 0, early1 = 0, early2 = 0, early3 = 0;        // physical pages of a chunk's first four pages, from the work list
     bool q_ok;
-    if (a.decode) {
+    if constexpr (DECODE) {
         DecodeWork w;
         int which;
         const int hc = (R + 31) / 32;
@@ -91,8 +91,8 @@ __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_plain_mfma_kernel(AttnA
         first_head = g * R + (which % hc) * 32;
         n_rows = min(32, R - (which % hc) * 32);
         work_index = seq * (a.G * hc) + which;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) early[i] = w.phys[i];
+        early0 = __builtin_amdgcn_readfirstlane(w.phys[0]), early1 = __builtin_amdgcn_readfirstlane(w.phys[1]);
+        early2 = __builtin_amdgcn_readfirstlane(w.phys[2]), early3 = __builtin_amdgcn_readfirstlane(w.phys[3]);
         tok = seq, qpos = qpos_first = w.qpos, hi = w.qpos;
         page_lo = w.page_lo, page_hi = w.page_hi;
         first_tile = 2 * w.first_page, kept_tiles = 2 * w.kept_pages;
@@ -138,12 +138,12 @@ __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_plain_mfma_kernel(AttnA
     const size_t k_page_elems = (size_t)a.G * PAGE_TOKENS * D, v_page_elems = (size_t)a.G * PAGE_TOKENS * DV;
 
     const int tile_hi = min(2 * page_hi, hi / 32 + 1);       // tiles of 32 keys: this wave takes tile_lo, tile_lo + PLAIN_WAVES, ... below tile_hi
-    const bool keys_in_turn = !a.waves_take_heads;           // the waves share one head's keys
+    const bool keys_in_turn = DECODE || !a.waves_take_heads;           // the waves share one head's keys
     const int tile_step = keys_in_turn ? PLAIN_WAVES : 1;
     // with a window or stretches, the tile of 32 keys that holds the oldest key any query of this wave sees; kept first
     // tokens: their tiles come ahead of those (tiles are counted as counted_page counts, from first_tile - kept_tiles on)
     const int oldest = first_seen(a, qpos_first), my_oldest = first_seen(a, qpos);
-    const int tile_lo = (a.keep_first == 0 ? max(2 * page_lo, oldest / 32) : a.decode ? 2 * page_lo : first_tile - kept_tiles) + (keys_in_turn ? wave : 0);
+    const int tile_lo = (a.keep_first == 0 ? max(2 * page_lo, oldest / 32) : DECODE ? 2 * page_lo : first_tile - kept_tiles) + (keys_in_turn ? wave : 0);
     // two sets of operands in turn: the loads of the tile after this one are queued before this
     // tile's products and stay there (the scheduler may not move them past the barrier), and the
     // page of the tile after that is looked up meanwhile
@@ -152,26 +152,31 @@ __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_plain_mfma_kernel(AttnA
         const int t = counted_page(counted, first_tile, kept_tiles);
         load_tile<D, DV>(ops, kbase + (size_t)phys * k_page_elems, vbase + (size_t)phys * v_page_elems, t & 1, lane);
     };
+    // (the same in every lane: numbers in scalar registers, and a load of the table that no vector load is waited for with)
+    // (values, chosen between before the branch: of variables read in either branch the compiler makes one read
+    // through a chosen address, from private memory)
     auto page_of = [&](int t) {
-        if (t >= tile_hi) return 0;
-        const int nth = t / 2 - page_lo;
-        if (a.decode && nth < 4) return nth < 2 ? (nth < 1 ? early[0] : early[1]) : nth < 3 ? early[2] : early[3];      // came with the entry: no trip to memory
-        return pt[(counted_page(t, first_tile, kept_tiles) / 2) % a.ring_pages];
+        const int nth = t / 2 - page_lo, e0 = early0, e1 = early1, e2 = early2, e3 = early3;
+        int page = nth < 2 ? (nth < 1 ? e0 : e1) : nth < 3 ? e2 : e3;      // came with the entry: no trip to memory
+        if (t >= tile_hi) page = 0;
+        else if (!DECODE || nth >= 4) page = pt[(counted_page(t, first_tile, kept_tiles) / 2) % a.ring_pages];
+        return __builtin_amdgcn_readfirstlane(page);
     };
-    // a tile's 16 biases of a lane, in base-2 units: asked for before the next tile's operands, because
-    // loads come back in the order they were queued and the softmax must not wait for those too
+    // a tile's 16 biases of a lane: asked for before the next tile's operands, because loads come back in
+    // the order they were queued and the softmax must not wait for those too (and nothing is made of them here, or
+    // the operands would wait for them)
     auto load_bias = [&](int t, float (&bv)[16]) {
         const int key0 = 32 * counted_page(t, first_tile, kept_tiles);
         if (!bias || t >= tile_hi) {
 #pragma unroll
             for (int e = 0; e < 16; ++e) bv[e] = 0.f;
         } else if (qpos_first - (key0 + 31) >= last_row) {      // wave-uniform: every pair of the tile is beyond the table
-            const float far_bias = bias[last_row] * LOG2E;
+            const float far_bias = bias[last_row];
 #pragma unroll
             for (int e = 0; e < 16; ++e) bv[e] = far_bias;
         } else {
 #pragma unroll
-            for (int e = 0; e < 16; ++e) bv[e] = bias[min(max(qpos - (key0 + key_of_elem(e, h)), 0), last_row)] * LOG2E;
+            for (int e = 0; e < 16; ++e) bv[e] = bias[min(max(qpos - (key0 + key_of_elem(e, h)), 0), last_row)];
         }
     };
     auto attend = [&](const TileOperands<D, DV>& ops, int t, const float (&bv)[16]) {
@@ -187,7 +192,7 @@ __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_plain_mfma_kernel(AttnA
             for (int e = 0; e < 16; ++e) S[e] = cap2 - 2.f * cap2 * __builtin_amdgcn_rcpf(1.f + exp2_flushing(S[e] * scale_cap));
         } else {
 #pragma unroll
-            for (int e = 0; e < 16; ++e) S[e] = fmaf(S[e], scale2, bv[e]);
+            for (int e = 0; e < 16; ++e) S[e] = fmaf(S[e], scale2, bv[e] * LOG2E);
         }
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
@@ -218,21 +223,27 @@ __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_plain_mfma_kernel(AttnA
             for (int ks = 0; ks < 2; ++ks) O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ops.V[dt][ks], Pf[ks], O[dt], 0, 0, 0);
         }
     };
-    if (tile_lo < tile_hi) fetch(A, tile_lo, page_of(tile_lo));
-    int phys_b = page_of(tile_lo + tile_step), phys_a = 0;
+    // A prompt's waves ask for a tile behind their last one too, which is that one again: where a branch may have asked for
+    // nothing, the compiler waits for all there is before a tile's products, and the next tile's operands with it.
+    // (A decode step's few tiles would only wait for that one at the end.)
+    int phys_a = page_of(tile_lo);
+    if (tile_lo < tile_hi) fetch(A, tile_lo, phys_a);
+    int phys_b = page_of(tile_lo + tile_step);
     float bv[16];
     for (int t = tile_lo; t < tile_hi; t += 2 * tile_step) {
         const int tb = t + tile_step, ta = t + 2 * tile_step;
         load_bias(t, bv);
         __builtin_amdgcn_sched_barrier(0);
-        if (tb < tile_hi) fetch(B, tb, phys_b);
+        if (!DECODE) fetch(B, tb < tile_hi ? tb : t, tb < tile_hi ? phys_b : phys_a);
+        else if (tb < tile_hi) fetch(B, tb, phys_b);
         phys_a = page_of(ta);
         __builtin_amdgcn_sched_barrier(0);
         attend(A, t, bv);
         if (tb >= tile_hi) break;
         load_bias(tb, bv);
         __builtin_amdgcn_sched_barrier(0);
-        if (ta < tile_hi) fetch(A, ta, phys_a);
+        if (!DECODE) fetch(A, ta < tile_hi ? ta : tb, ta < tile_hi ? phys_a : phys_b);
+        else if (ta < tile_hi) fetch(A, ta, phys_a);
         phys_b = page_of(ta + tile_step);
         __builtin_amdgcn_sched_barrier(0);
         attend(B, tb, bv);
@@ -311,8 +322,8 @@ __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_plain_mfma_kernel(AttnA
             o = make_float2(fmaf(o.x, mine_k, v.x * other_k), fmaf(o.y, mine_k, v.y * other_k));
             m = m_new;
         }
-        const int hq = a.decode ? first_head + q : first_head, row = a.decode ? seq : first_tok + q;
-        if (a.decode && n_chunks > 1) {
+        const int hq = DECODE ? first_head + q : first_head, row = DECODE ? seq : first_tok + q;
+        if (DECODE && n_chunks > 1) {
             float* po = a.partial + (((size_t)seq * a.H + hq) * a.max_splits + split) * (DV + 2);
             m = m > 0.5f * NEG_BIG ? m * LN2 : NEG_BIG;       // the merge works with e-based exponents
             if (a.chunks_done) {             // read back by another workgroup of this launch
@@ -328,7 +339,7 @@ __global__ __launch_bounds__(64 * PLAIN_WAVES) void attn_plain_mfma_kernel(AttnA
             store(row, hq, c, gated(gate, c, o.x * inv), gated(gate, c + 1, o.y * inv));
         }
     }
-    if (!a.decode || n_chunks <= 1 || !a.chunks_done) return;       // (uniform over the workgroup)
+    if (!DECODE || n_chunks <= 1 || !a.chunks_done) return;       // (uniform over the workgroup)
     // The workgroup that finishes a sequence's last chunk reads all of them back and writes the
     // output, so that the sum does not depend on who it was; see
     // attn_decode_mfma_kernel for why single coherent accesses and no fence.
@@ -404,27 +415,32 @@ extern "C" int picolm_attn_plain_mfma_takes(int d, int dv) {
 }
 extern "C" int picolm_attn_plain_mfma_tile_rows(void) { return 32; }
 
-template <int D, int DV>
+template <int D, int DV, bool DECODE>
 static int launch_sized(const AttnArgs& a, dim3 grid, hipStream_t stream) {
-    const int rows = a.decode ? (a.H / a.G < 32 ? a.H / a.G : 32) : 32;
+    const int rows = DECODE ? (a.H / a.G < 32 ? a.H / a.G : 32) : 32;
     const size_t lds = a.waves_take_heads ? 0 : sizeof(float) * PLAIN_WAVES * rows * (DV + 4);       // at most 66 KB
     constexpr size_t most = sizeof(float) * PLAIN_WAVES * 32 * (DV + 4);
     static bool raised = most <= 48 * 1024;
     if (!raised) {
-        hipError_t e = hipFuncSetAttribute((const void*)attn_plain_mfma_kernel<D, DV>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)most);
+        hipError_t e = hipFuncSetAttribute((const void*)attn_plain_mfma_kernel<D, DV, DECODE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)most);
         PICOLM_REQUIRE(e == hipSuccess, "attn_plain_mfma: cannot raise the LDS limit to %zu: %s", most, hipGetErrorString(e));
         raised = true;
     }
-    attn_plain_mfma_kernel<D, DV><<<grid, 64 * PLAIN_WAVES, lds, stream>>>(a);
+    attn_plain_mfma_kernel<D, DV, DECODE><<<grid, 64 * PLAIN_WAVES, lds, stream>>>(a);
     PICOLM_LAUNCH_CHECK("attn_plain_mfma");
     return 0;
 }
-template <int D>
+template <int D, bool DECODE>
 static int launch_dv(const AttnArgs& a, int dv, dim3 grid, hipStream_t stream) {
-    return dv == 64 ? launch_sized<D, 64>(a, grid, stream) : dv == 96 ? launch_sized<D, 96>(a, grid, stream) : launch_sized<D, 128>(a, grid, stream);
+    return dv == 64   ? launch_sized<D, 64, DECODE>(a, grid, stream)
+           : dv == 96 ? launch_sized<D, 96, DECODE>(a, grid, stream)
+                      : launch_sized<D, 128, DECODE>(a, grid, stream);
 }
+template <bool DECODE>
 static int launch(const AttnArgs& a, int dv, dim3 grid, hipStream_t stream) {
-    return a.d == 64 ? launch_dv<64>(a, dv, grid, stream) : a.d == 96 ? launch_dv<96>(a, dv, grid, stream) : launch_dv<128>(a, dv, grid, stream);
+    return a.d == 64   ? launch_dv<64, DECODE>(a, dv, grid, stream)
+           : a.d == 96 ? launch_dv<96, DECODE>(a, dv, grid, stream)
+                       : launch_dv<128, DECODE>(a, dv, grid, stream);
 }
 
 int check_attn_sizes(const char* who, int H, int G, int d, int max_pages, int ring_pages);
@@ -471,7 +487,7 @@ extern "C" int picolm_attn_prefill_plain_mfma(const void* q, const void* k_pages
     // (measured at 2,048 tokens: a head a wave is faster once its workgroups fill the 256 CUs, 0.39 against 0.47 ms
     // for two layers of 16 heads; with 8 heads the keys in turn are, 0.40 against 0.57 ms)
     a.waves_take_heads = (H / G) % PLAIN_WAVES == 0 && (int64_t)n_tiles * (H / PLAIN_WAVES) >= 256;
-    return launch(a, dv, dim3(n_tiles, a.waves_take_heads ? H / PLAIN_WAVES : H), stream);
+    return launch<false>(a, dv, dim3(n_tiles, a.waves_take_heads ? H / PLAIN_WAVES : H), stream);
 }
 
 extern "C" int picolm_attn_decode_plain_mfma(const void* q, const void* k_pages, const void* v_pages, void* out, float* partial, int n_seq,
@@ -491,7 +507,7 @@ extern "C" int picolm_attn_decode_plain_mfma(const void* q, const void* k_pages,
     int dv;
     if (fill_extras("attn_decode_plain_mfma", a, x, dv)) return -1;
     a.chunks_done = max_splits > 1 ? chunks_done : nullptr;
-    const int rc = launch(a, dv, dim3(n_chunks * G * hc), stream);
+    const int rc = launch<true>(a, dv, dim3(n_chunks * G * hc), stream);
     if (rc) return rc;
     return max_splits > 1 && !a.chunks_done ? picolm_attn_merge_launch(a, PICOLM_BF16, n_seq, stream) : 0;
 }

@@ -41,6 +41,14 @@ def code_object_metadata(elf, msgpack):
     return {}
 
 
+def test_plain_page_attention_stays_in_registers():
+    """No private memory: a page looked up there is a wait for everything that is on its way."""
+    kernels = {n: k for n, k in kernels_metadata().items() if "attn_plain_mfma_kernel" in n}
+    assert len(kernels) == 18
+    for name, k in kernels.items():
+        assert k[".private_segment_fixed_size"] == 0 and k[".vgpr_spill_count"] == 0, name
+
+
 def test_shared_rows_begin_at_16_bytes():
     """Rows in dynamic LDS lie behind a kernel's fixed part, and are read and written 16 bytes at a time."""
     for name, k in kernels_metadata().items():
