@@ -67,6 +67,33 @@ struct Sums {
 #pragma unroll
         for (int e = 0; e < 4; ++e) Operand<float>::multiply(a, b, part[e], e);
     }
+    // A block on the diagonal of a lower triangle, whose zeros above it meet tokens that come later: a number of theirs that is
+    // not finite must not reach the rows before.  (Where there is one, the block's finite part goes through the MFMAs, and
+    // the rest to the rows from its token on.)
+    __device__ __forceinline__ void add_lower(const f32x4& a, const f32x4& b) {
+        bool fine = true;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) fine = fine && __builtin_isfinite(b[e]);
+        if (__all(fine)) {
+            add(a, b);
+            return;
+        }
+        f32x4 finite;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) finite[e] = __builtin_isfinite(b[e]) ? b[e] : 0.f;
+        add(a, finite);
+        const int lane = threadIdx.x % 64, col = lane % 16, q = lane / 16;
+        for (int jq = 0; jq < 4; ++jq)
+#pragma unroll
+            for (int je = 0; je < 4; ++je) {                // token 4 jq + je of the block
+                const float x = __shfl(b[je], 16 * jq + col, WAVE);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float factor = __shfl(a[je], 16 * jq + 4 * q + e, WAVE);
+                    if (!__builtin_isfinite(x) && 4 * q + e >= 4 * jq + je) part[0][e] += factor * x;
+                }
+            }
+    }
     __device__ __forceinline__ f32x4 total() const { return (part[0] + part[1]) + (part[2] + part[3]); }
 };
 
@@ -183,7 +210,7 @@ __global__ __launch_bounds__(256) void state_chunk_prepare_kernel(StateChunks a)
                 for (int e = 0; e < 4; ++e) b[e] = X[(16 * k + 4 * q + e) * SC_LD + 16 * J + r16];
                 ys.add(*(const f32x4*)(T + (16 * I + r16) * SC_LD + 16 * k + 4 * q), b);
             }
-            xs.add(*(const f32x4*)(X + (16 * I + r16) * SC_LD + 16 * I + 4 * q), ys.total());   // (rows 4q + e of the one are the operand's)
+            xs.add_lower(*(const f32x4*)(X + (16 * I + r16) * SC_LD + 16 * I + 4 * q), ys.total());   // (rows 4q + e of the one are the operand's)
             const f32x4 x = xs.total();
 #pragma unroll
             for (int e = 0; e < 4; ++e) X[(16 * I + 4 * q + e) * SC_LD + 16 * J + r16] = -x[e];
@@ -208,7 +235,8 @@ __global__ __launch_bounds__(256) void state_chunk_prepare_kernel(StateChunks a)
             Sums t;
             t.clear();
 #pragma unroll
-            for (int J = 0; J <= I; ++J) t.add(*(const f32x4*)(X + (16 * I + r16) * SC_LD + 16 * J + 4 * q), b[J]);
+            for (int J = 0; J < I; ++J) t.add(*(const f32x4*)(X + (16 * I + r16) * SC_LD + 16 * J + 4 * q), b[J]);
+            t.add_lower(*(const f32x4*)(X + (16 * I + r16) * SC_LD + 16 * I + 4 * q), b[I]);
             o[I] = t.total();
         }
         float* to = scratch + SC_LEN + (keys ? 0 : KD) + c;
@@ -315,7 +343,8 @@ __global__ __launch_bounds__(256) void state_chunk_walk_kernel(StateChunks a) {
         for (int v = 0; v < VT; ++v) {
 #pragma unroll
             for (int g = 0; g < 4; ++g)
-                if (g <= wave) os[v].add(x.af[g], *(const f32x4*)(Ut + (16 * v + r16) * SC_LD + 16 * g + 4 * q));
+                if (g < wave) os[v].add(x.af[g], *(const f32x4*)(Ut + (16 * v + r16) * SC_LD + 16 * g + 4 * q));
+                else if (g == wave) os[v].add_lower(x.af[g], *(const f32x4*)(Ut + (16 * v + r16) * SC_LD + 16 * g + 4 * q));
             // (St has been read by every wave; a wave reads and writes its own rows of it here)
 #pragma unroll
             for (int m = 0; m < KT; ++m) {

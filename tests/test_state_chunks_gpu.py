@@ -108,3 +108,25 @@ def test_decays_of_nought_and_strong_ones_in_chunks():
         x = Scan(rule, 4, 2, 128, 64, [130])
         x.raw[20, 3:7], x.raw[70:90, 3:7], x.A_log[1] = 200.0, 30.0, 3.0
         assert max(distances(x.run(), x.reference())) < 2e-6
+
+
+# a token in the middle of a block of 16, a block's last, a chunk's first and its last but one, the sequence's last
+@pytest.mark.parametrize("rule,H,G,kd,vd", SIZES)
+@pytest.mark.parametrize("at", [37, 47, 64, 126, 136])
+def test_what_is_no_number_reaches_no_token_before_it(rule, H, G, kd, vd, at):
+    """Queries, keys, values, strengths and decays: outputs before the token are those of a sequence without it, to the bit, and
+    no number where the walk has none."""
+    inf, nan = float("inf"), float("nan")
+    x = Scan(rule, H, G, kd, vd, [137])
+    clean = x.run()[0]
+    for column, value in ((5, nan), (G * kd + 3, inf), (G * kd + kd - 1, nan), (2 * G * kd + 7, inf), (2 * G * kd + vd + 1, -inf), (("raw", 3), nan),
+                          (("raw", 3 + H), nan)):
+        y = Scan(rule, H, G, kd, vd, [137])
+        if isinstance(column, tuple):
+            y.raw[at, column[1]] = value
+        else:
+            y.qkv[at, column] = value
+        (got, state), (walked, walked_state) = y.run(), y.run(chunked=False)
+        assert torch.equal(got[:at], clean[:at]), (column, value)
+        assert torch.equal(got.isfinite(), walked.isfinite()) and torch.equal(state.isfinite(), walked_state.isfinite()), (column, value)
+        assert not got[at].isfinite().all()
