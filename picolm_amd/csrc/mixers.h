@@ -94,7 +94,7 @@ int picolm_call_short_conv(void* user, const picolm_step_view* v);
 // A matrix state S [key_dim][value_dim] per head and sequence, walked over the step's tokens in
 // order, kept in float in the slot's state.  With per-token decay a and strength w (both per head):
 //   rule 0 (outer product):  S <- a S + w k v^T;                      o = S^T q + skip v
-//   rule 1 (delta rule):     S <- a S;  S <- S + k (w (v - S^T k))^T;  o = S^T q
+//   rule 1 (delta rule):     S <- a S;  S <- S + k (w (v - S^T k))^T;  o = S^T q + skip v
 //   a = exp(-exp(A_log) softplus(raw_a + dt_bias));  w = softplus(raw_w + dt_bias) (rule 0) or
 //   sigmoid(raw_w) (rule 1).  unit_qk: q and k are first made unit vectors per head
 //   (x / sqrt(sum x^2 + unit_eps)); q is multiplied by q_scale.

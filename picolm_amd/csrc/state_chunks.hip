@@ -292,7 +292,7 @@ __global__ __launch_bounds__(256) void state_chunk_walk_kernel(StateChunks a) {
 #pragma unroll
             for (int v = 0; v < VT; ++v) {
                 const int col = cb * VB + 16 * v + r16;
-                x.vv[v][e] = RULE == 0 ? qkv[(size_t)t * a.qkv_stride + a.v_off + (size_t)head * vd + col] : 0.f;
+                x.vv[v][e] = RULE == 0 || a.skip ? qkv[(size_t)t * a.qkv_stride + a.v_off + (size_t)head * vd + col] : 0.f;
                 x.u0[v][e] = RULE == 0 ? w : scratch[t * srow + SC_LEN + KD + col];
             }
         }

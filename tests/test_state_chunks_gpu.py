@@ -10,11 +10,12 @@ DEV = "cuda:0"
 
 
 class Scan:
-    def __init__(self, rule, heads, key_heads, kd, vd, lengths, seed=0, slow=True):
+    def __init__(self, rule, heads, key_heads, kd, vd, lengths, seed=0, slow=True, skips=None):
         gen = torch.Generator(device=DEV).manual_seed(seed + kd + vd)
         randn = lambda *s: torch.randn(*s, generator=gen, device=DEV)
         T = sum(lengths)
         self.rule, self.H, self.G, self.kd, self.vd, self.lengths = rule, heads, key_heads, kd, vd, lengths
+        self.skips = rule == 0 if skips is None else skips          # outputs take a share of the value
         self.stride = 2 * key_heads * kd + heads * vd + 4
         self.qkv, self.raw = randn(T, self.stride), randn(T, 2 * heads + 3)
         self.state = randn(len(lengths), heads, kd, vd)
@@ -33,7 +34,7 @@ class Scan:
         qkv, aw, out = self.qkv.clone(), torch.empty(T, 2 * H, device=DEV), torch.full((T, H * vd), 9.0, device=DEV)
         scratch = torch.full((T, H * (68 + (kd + vd if self.rule else 0))), float("nan"), device=DEV)
         args = StateScanArgs(self.rule, H, G, kd, vd, self.raw.shape[1], 3, 3 + H, self.stride, 0, G * kd, 2 * G * kd, self.A_log.data_ptr(),
-                             self.bias.data_ptr(), None if self.rule else self.skip.data_ptr(), self.rule, 1e-6, kd ** -0.5, 8)
+                             self.bias.data_ptr(), self.skip.data_ptr() if self.skips else None, self.rule, 1e-6, kd ** -0.5, 8)
         v = P.StepView()
         v.struct_bytes, v.dtype, v.rows, v.n_tokens, v.n_seq = ctypes.sizeof(P.StepView), 0, T, T, n
         v.is_decode = int(max(self.lengths) == 1)
@@ -70,7 +71,7 @@ class Scan:
                 S = a[t, :, None, None] * S
                 u = w[t, :, None] * (v[t] - (S * k[t, :, :, None]).sum(1) if self.rule else v[t])
                 S = S + k[t, :, :, None] * u[:, None, :]
-                outs.append((S * q[t, :, :, None]).sum(1) + (0.0 if self.rule else self.skip.double()[:, None] * v[t]))
+                outs.append((S * q[t, :, :, None]).sum(1) + (self.skip.double()[:, None] * v[t] if self.skips else 0.0))
                 t += 1
             states.append(S)
         return torch.stack(outs).reshape(-1, H * vd), torch.stack(states)
@@ -130,3 +131,11 @@ def test_what_is_no_number_reaches_no_token_before_it(rule, H, G, kd, vd, at):
         assert torch.equal(got[:at], clean[:at]), (column, value)
         assert torch.equal(got.isfinite(), walked.isfinite()) and torch.equal(state.isfinite(), walked_state.isfinite()), (column, value)
         assert not got[at].isfinite().all()
+
+
+# a prompt in chunks, one that is walked, a decode step
+@pytest.mark.parametrize("lengths", [[70, 16], [15], [1, 1, 1]])
+@pytest.mark.parametrize("rule,skips", [(1, True), (0, False)])
+def test_either_rule_with_and_without_a_share_of_the_value(rule, skips, lengths):
+    x = Scan(rule, 4, 2, 128, 64, lengths, skips=skips)
+    assert max(distances(x.run(), x.reference())) < 1e-6
