@@ -1171,9 +1171,11 @@ static int grouped_product(const bf16_t* a, const int32_t* plan, void* out, cons
 
 #define GM_FROM_ROWS 64      // rows of a step from which the matrix cores take the experts
 
-// What either kind of kernels that read an expert's weights once needs: bfloat16 throughout, 16-byte aligned buffers and rows
+// What either kind of kernels that read an expert's weights once needs: bfloat16 throughout, 16-byte aligned buffers and rows,
+// and room for the pairs' outputs
 static bool reads_weights_once(const picolm_routed_experts_args* a, const picolm_step_view* v, int widths_in) {
     return v->dtype == PICOLM_BF16 && a->weight_dt == PICOLM_BF16 && a->width % widths_in == 0 && a->ff % widths_in == 0 && v->extra[2] &&
+           v->extra_row_bytes[2] >= (int64_t)a->top * a->width * 4 &&
            (((uintptr_t)v->in | (uintptr_t)v->out | (uintptr_t)v->extra[1] | (uintptr_t)v->extra[2] | (uintptr_t)a->gate | (uintptr_t)a->up |
              (uintptr_t)a->down) & 15) == 0;
 }
@@ -1219,7 +1221,6 @@ extern "C" int picolm_call_routed_experts(void* user, const picolm_step_view* v)
     float* act = (float*)v->extra[1];
     const bool chains = takes_chains(a, v);
     if (chains || streams_experts(a, v)) {
-        PICOLM_REQUIRE(v->extra_row_bytes[2] >= (int64_t)top * D * 4, "routed_experts: scratch rows too short for the pairs' outputs");
         float* y = (float*)v->extra[2];
         int rc = (chains ? launch_expert_chains<true> : launch_expert_stream<true>)(v->in, picks, act, (const bf16_t*)a->gate, (const bf16_t*)a->up, E, top, v->rows, D, F, xa, v->stream);
         if (rc) return rc;
