@@ -578,7 +578,10 @@ __global__ __launch_bounds__(256) void grouped_tile_kernel(const bf16_t* __restr
 // out[row] (+)= sum_k w[row][k] y[row][k], in the order of the picks; four columns a thread (D is a
 // multiple of four), so that a row's picks are asked for in one trip and a step of few rows has a
 // workgroup for every 1,024 columns
+// (out and the inputs need not begin at 16 bytes: in a prompt's step nothing else asks for that)
 #define GSUM_AT_ONCE 8
+typedef __attribute__((ext_vector_type(4), aligned(4))) float floats_anywhere;
+typedef __attribute__((ext_vector_type(2), aligned(2))) unsigned bf16_four_anywhere;
 __global__ __launch_bounds__(256) void grouped_sum_kernel(const float* __restrict__ y, const int32_t* __restrict__ picks, float* __restrict__ out,
                                                           int E, int top, int D, int adds, const bf16_t* __restrict__ h, int identity,
                                                           int plain_sum) {
@@ -587,17 +590,17 @@ __global__ __launch_bounds__(256) void grouped_sum_kernel(const float* __restric
     if (d >= D) return;
     const int32_t* ids = picks + row * 2 * top;
     const float* w = (const float*)(ids + top);
-    float4* o = (float4*)(out + row * D + d);
-    float4 total = make_float4(0.f, 0.f, 0.f, 0.f);
-    const float4 before = adds ? *o : total;
+    floats_anywhere* o = (floats_anywhere*)(out + row * D + d);
+    floats_anywhere total = {0.f, 0.f, 0.f, 0.f}, before = total, input = total;
+    if (adds) before = *o;
     for (int k0 = 0; k0 < top; k0 += GSUM_AT_ONCE) {
-        float4 part[GSUM_AT_ONCE];
+        floats_anywhere part[GSUM_AT_ONCE];
         float wk[GSUM_AT_ONCE];
 #pragma unroll
         for (int i = 0; i < GSUM_AT_ONCE; ++i) {
             const int k = min(k0 + i, top - 1), e = ids[k];
             wk[i] = k0 + i < top && e >= 0 && e < E ? (plain_sum ? 1.f : w[k]) : 0.f;
-            if (k0 + i < top) part[i] = *(const float4*)(y + (row * top + k) * D + d);       // (of a pick without an expert: not used)
+            if (k0 + i < top) part[i] = *(const floats_anywhere*)(y + (row * top + k) * D + d);       // (of a pick without an expert: not used)
         }
 #pragma unroll
         for (int i = 0; i < GSUM_AT_ONCE; ++i)
@@ -609,15 +612,14 @@ __global__ __launch_bounds__(256) void grouped_sum_kernel(const float* __restric
             }
     }
     const float same = identity > 0 ? identity_weight(ids, w, top, E, identity) : 0.f;
-    float4 input = make_float4(0.f, 0.f, 0.f, 0.f);
     if (same != 0.f) {
-        const uint2 hv = *(const uint2*)(h + row * D + d);
-        input = make_float4(__uint_as_float(hv.x << 16), __uint_as_float(hv.x & 0xffff0000u), __uint_as_float(hv.y << 16),
-                            __uint_as_float(hv.y & 0xffff0000u));
+        const bf16_four_anywhere hv = *(const bf16_four_anywhere*)(h + row * D + d);
+        input = floats_anywhere{__uint_as_float(hv.x << 16), __uint_as_float(hv.x & 0xffff0000u), __uint_as_float(hv.y << 16),
+                                __uint_as_float(hv.y & 0xffff0000u)};
     }
     // (as expert_down_kernel adds up, to the bit)
     const auto sum = [&](float b, float t, float x) { return b + t + (same != 0.f ? same * x : 0.f); };
-    *o = make_float4(sum(before.x, total.x, input.x), sum(before.y, total.y, input.y), sum(before.z, total.z, input.z), sum(before.w, total.w, input.w));
+    *o = floats_anywhere{sum(before.x, total.x, input.x), sum(before.y, total.y, input.y), sum(before.z, total.z, input.z), sum(before.w, total.w, input.w)};
 }
 
 // ---- the same for a few rows, the experts' weights read once, to the bit -----------------------------------

@@ -20,3 +20,13 @@ def test_grouped_experts(E, D, F, rows, top):
 def test_grouped_experts_identity_picks_clamps_and_weights_on_the_input():
     assert check(Experts(4, 128, 192, identity=3), 300, 5)[0] < 4e-3
     assert check(Experts(4, 128, 192, act=1, weight_on_input=1), 300, 3)[0] < 4e-3
+
+
+def test_rows_of_a_prompt_need_not_begin_at_16_bytes():
+    import torch
+    x = Experts(4, 128, 192, identity=1)
+    h = torch.randn(300, 128, generator=x.gen, device="cuda:0").bfloat16()
+    ids, w, words = x.picks(300, 3)
+    aligned = x.run(h, words, 3, torch.ones(300, 128, device="cuda:0"), True)
+    room = torch.ones(300 * 128 + 1, device="cuda:0")
+    assert torch.equal(x.run(h, words, 3, room[1:].view(300, 128), True), aligned) and float(room[0]) == 1.0
