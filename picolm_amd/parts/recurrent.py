@@ -52,11 +52,18 @@ def _check_sizes(key_dim: int, taps: int) -> None:
         raise ValueError(f"a convolution of {taps} taps: the kernel takes 1 to {SHORT_CONV_MAX_TAPS}")
 
 
+# The most that a token's row of the chunks' scratch may take: 4 GiB in a prefill step of 16,384 tokens, as the
+# scratch of the walk in chunks has for its limit (16 heads of 128 x 128 with the delta rule: 20.7 KB, 340 MB a step).
+CHUNK_ROW_BYTES = 1 << 18
+
+
 def _chunk_rows(b, heads: int, key_dim: int, value_dim: int, more: int) -> list:
-    """Scratch rows with which state_scan takes a prompt in chunks (sizes as csrc/state_chunks.hip has them)."""
-    if key_dim not in (64, 128) or value_dim % 16:
+    """Scratch rows with which state_scan takes a prompt in chunks (sizes as csrc/state_chunks.hip has them); without
+    them it is walked."""
+    floats = heads * (64 + more + 4)
+    if key_dim not in (64, 128) or value_dim % 16 or 4 * floats > CHUNK_ROW_BYTES:
         return []
-    return [b.buffer("scan.chunks", heads * (64 + more + 4), torch.float32)]
+    return [b.buffer("scan.chunks", floats, torch.float32)]
 
 
 class GatedDeltaRule(Mixer):
