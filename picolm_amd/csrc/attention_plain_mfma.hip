@@ -18,9 +18,12 @@
 //   decode : a workgroup takes one entry of the step's work list and one KV group; its columns are
 //            the group's query heads (32 at a time).  The chunk's first four pages come with the
 //            entry.  The workgroup that finishes a sequence's last chunk combines them where the
-//            caller has counters (else the merge kernel of attention_generic.hip does).  A few
-//            hundred keys a chunk are latencies, not bytes: an attention of 16 heads over 1,000 to
-//            2,000 tokens took 10 to 13 us and its merge kernel 5 to 7; in one launch 11 to 15.
+//            caller has counters (else the merge kernel of attention_generic.hip does, with the
+//            same sums).  A few hundred keys a chunk are latencies, not bytes: an attention of 16 heads over
+//            1,000 to 2,000 tokens took 10 to 13 us and its merge kernel 5 to 7; in one launch 11.5 to 13
+//            (13 to 15 while the pages of a chunk lay in private memory).
+// A prompt is bound by its longest tiles' chain of keys (matrix cores 3 % busy): four prompts of 301 to 1,203 tokens, 16 heads of
+// 128 over 4 with a bias, 153 us a layer (194 with pages from private memory and biases multiplied as they came).
 // Statistics are float in the base-2 domain; the bias table is [H][bias_rows].
 #include "common.h"
 #include "api.h"

@@ -632,7 +632,7 @@ __global__ __launch_bounds__(256) void grouped_sum_kernel(const float* __restric
 // A pair's sums are those of the kernels above, to the bit: chain l of 64 adds the products of columns 8 l .. + 7 of
 // every 512, one after another, and the chains' sums meet by halves, quarters, ... of the 64.  A chain is a block of
 // v_mfma_f32_4x4x1_16b_f32, which does one FMA for each of four weight rows and four pairs in 16 chains: twice the rate of
-// the vector ALU.  (The bfloat16 MFMAs, four times as fast again, add several products up in an order of their own.  A
+// the vector ALU.  (The bfloat16 MFMAs, sixteen times as fast as these, add several products up in an order of their own.  A
 // step's pairs are few enough for the float ones, and with other sums than a workgroup per pair has, a router behind
 // them that is not sure of a pick decides otherwise.)
 // Which pairs share an expert changes no pair's result.
@@ -936,7 +936,8 @@ static int launch_expert_chains(const void* a, const int32_t* picks, float* out,
 // Bound by the experts' bytes: sixteen experts of 4,096 x 4,096 at 64 rows, two picked, 263 us with the adding
 // kernel where the weights of the experts picked take 248 at 6.5 TB/s; 64 of 1,408 x 2,048, six picked, 213 us, floor 170.
 #define ES_MOST_PAIRS 512      // pairs of one expert that a workgroup lists (a row picks an expert once)
-// eight floats as three bfloat16 chunks: x = hi + mid + lo (a number that is not finite lies in hi alone)
+// eight floats as three bfloat16 chunks: x = hi + mid + lo (a number that is not finite lies in hi alone), as in Henry, Tang and
+// Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision Computations", 2019
 __device__ __forceinline__ void split_chunk(const f32x4& x0, const f32x4& x1, bf16x8& hi, bf16x8& mid, bf16x8& lo) {
     u32x4 h, m, l;
 #pragma unroll

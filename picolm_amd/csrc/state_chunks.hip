@@ -10,14 +10,15 @@
 // The delta rule's u is a triangular system, (I + T) U = diag(w) V - diag(w p) K S0 with T_tj = w_t D_tj (k_j . k_t):
 // X = (I + T)^-1 comes from its blocks of 16 (each turned over column by column; the blocks below the
 // diagonal, -X_II sum_K T_IK X_KJ, are products), and U = X diag(w) V - (X diag(w p) K) S0.  Every factor is a product
-// of decays; nothing is divided by one.  Two kernels:
+// of decays; nothing is divided by one.  (The chunked form of the delta rule is that of Yang, Wang, Zhang, Shen and Kim, "Parallelizing
+// Linear Transformers with the Delta Rule over Sequence Length", 2024; inverting a unit lower triangle by blocks is textbook.)  Two kernels:
 //   prepare  per (sequence, chunk, head), side by side: A_ij = D_ij (q_i . k_j), and for the delta rule
 //            -X diag(w p) K and X diag(w) V; p and D_C.  A token's share of them is a row of scratch memory.
 //   walk     per (sequence, head, 16 or 32 value columns), chunk by chunk in order: U, the outputs, and the next
 //            state, which stays in LDS.
 // Bound by the walk's chain, 8.7 us a chunk: three products (3 us of the matrix cores), two meetings of the waves, and the
 // chunk's operands from L2 and beyond (115 KB; asked for a chunk ahead it was no faster, and where two
-// workgroups share a CU slower: 204 against 160 us).  Four prompts of 301 to 1,203 tokens: a layer of 16 heads of 128 x 128
+// workgroups share a CU slower: 204 against 160 us).  (Counted: the matrix cores 20 to 30 % busy, 42 % of the LDS cycles bank conflicts.)  Four prompts of 301 to 1,203 tokens: a layer of 16 heads of 128 x 128
 // with the delta rule 253 us (the walk in chunks of its own, in mixers.hip, 1,087), of 64 heads of 128 x 64 with outer
 // products 230 (1,160); a decode step of four sequences 7.9 and 6.9 us (26.6 and 22.8 with the kernel that prepares).
 #include "mixers.h"

@@ -74,8 +74,8 @@ def check(x, rows, top, adds=False, seed=0):
     return float((got - want).norm() / want.norm()), float((got - want).abs().max() / want.abs().max())
 
 
-# 16 pairs of an expert a tile, 16, 32 and 64 at a time, more than 64; fewer pairs than experts; one expert; widths that
-# are one line, no power of two, and less than the four waves' lines
+# up to four, eight and 16 pairs of an expert at a time and more than that, from 64 rows on tiles of 16 pairs, 16, 32 and 64 at a
+# time; fewer pairs than experts; one expert; widths that are one line, no power of two, and less than the four waves' lines
 @pytest.mark.parametrize("E,D,F", [(1, 64, 64), (8, 2048, 2048), (3, 192, 320), (40, 320, 192), (2, 128, 1344)])
 @pytest.mark.parametrize("rows", [1, 2, 7, 16, 17, 33, 63, 64, 100, 255])
 def test_streamed_experts(E, D, F, rows):
@@ -83,7 +83,8 @@ def test_streamed_experts(E, D, F, rows):
     top = min(E, 2 if rows % 2 else 3)
     norm, worst = check(x, rows, top, adds=rows % 2 == 1)
     # exact products, float sums of up to 2,048 of them: a few roundings of 2^-24 each, with the hidden units' own; steps of
-    # 64 rows and more with many pairs an expert go through tiles that round the hidden units to eight bits (2^-9 each)
+    # 64 rows and more with many pairs an expert go through tiles that round the hidden units to eight bits (2^-9 each).  Which
+    # steps keep them in 32 bits is what the library promises, and said here again: a step that no longer did would fail
     streamed = rows < 64 or rows * top <= 20 * E
     assert norm < (2e-6 if streamed else 4e-3) and worst < (1e-5 if streamed else 2e-2), (E, D, F, rows, norm, worst)
 
