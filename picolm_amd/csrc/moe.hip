@@ -638,7 +638,7 @@ __global__ __launch_bounds__(256) void grouped_sum_kernel(const float* __restric
 // Which pairs share an expert changes no pair's result.
 // Bound by the experts' bytes: sixteen experts of 4,096 x 4,096 at 16 rows, two picked, 238 us with the adding
 // kernel where the weights of the experts picked take 201 at 6.5 TB/s (a workgroup per pair and 16 units, which
-// read an expert's weights for every pair of its own: 742); eight of 2,048 x 2,048 47.7 us, floor 31 (203).  From eight pairs
+// read an expert's weights for every pair of its own: 742); eight of 2,048 x 2,048 47.5 us, floor 31 (203).  From eight pairs
 // an expert on the MFMAs' time shows (48 rows: hidden units 45 us, 13 of them if nothing else ran; 16 rows: 31.6).
 #define EC_LISTED 1024         // pairs of the step of which a workgroup lists its expert's at a time
 typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
@@ -1183,7 +1183,7 @@ static bool reads_weights_once(const picolm_routed_experts_args* a, const picolm
              (uintptr_t)a->down) & 15) == 0;
 }
 // Below 64 rows every kernel gives a row the same bits, and the chains are the fastest that do: eight experts of 2,048 x
-// 2,048, two picked, 16 rows 47.7 us against 203 with a workgroup per pair, 32 rows 59 and 63 rows 86.  (The bfloat16 MFMAs
+// 2,048, two picked, 16 rows 47.5 us against 203 with a workgroup per pair, 32 rows 55 and 63 rows 83.  (The bfloat16 MFMAs
 // take 46 to 51 at any of these, in another order of sums.)
 static bool takes_chains(const picolm_routed_experts_args* a, const picolm_step_view* v) {
     return v->rows < GM_FROM_ROWS && a->experts <= 65535 && (int64_t)v->rows * a->top <= 65535 && reads_weights_once(a, v, 8);
